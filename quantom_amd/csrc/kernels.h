@@ -318,6 +318,13 @@ LIMA_DEV void local_role(const StepArgs& a, int c, char* lds) {
     }
     sync();
     double eb = 0, ea = 0, ed = 0;
+    // Energies of the terms that thread 0 of the reference's 128 evaluates, for its potE slot of the
+    // log: every 128th term, whatever this form's stride.  The thread of term 0 has them all.
+    double slot_b = 0, slot_a = 0, slot_d = 0;
+    auto count = [](double& sum, double& slot, int t, double e) {
+        sum += e;
+        slot += t % kCompoundBlock == 0 ? e : 0.0;
+    };
     const int b0 = a.bond_off[c], nb = a.bond_off[c + 1] - b0;
     const int a0 = a.angle_off[c], na = a.angle_off[c + 1] - a0;
     const int d0 = a.dih_off[c], nd = a.dih_off[c + 1] - d0;
@@ -325,17 +332,23 @@ LIMA_DEV void local_role(const StepArgs& a, int c, char* lds) {
     if (WAVE || p >= P) {
         for (int t = WAVE ? p : p - P; t < nb; t += P) {
             BondD bd = a.bonds[b0 + t];
-            pairbond(P3(bd.a0), P3(bd.a1), bd.b0, bd.kb, &rb[t * 2], &eb);
+            double e = 0;
+            pairbond(P3(bd.a0), P3(bd.a1), bd.b0, bd.kb, &rb[t * 2], &e);
+            count(eb, slot_b, t, e);
         }
         for (int t = WAVE ? p : p - P; t < na; t += P) {
             AngleD ad = a.angles[a0 + t];
-            anglebond(P3(ad.a0), P3(ad.a1), P3(ad.a2), ad.t0, ad.k, &ra[t * 3], &ea);
+            double e = 0;
+            anglebond(P3(ad.a0), P3(ad.a1), P3(ad.a2), ad.t0, ad.k, &ra[t * 3], &e);
+            count(ea, slot_a, t, e);
         }
     }
     if (a.enable_dihedrals && p < P) {
         for (int t = p; t < nd; t += P) {
             DihD dd = a.dihs[d0 + t];
-            dihedral(P3(dd.a0), P3(dd.a1), P3(dd.a2), P3(dd.a3), dd.p0, dd.k, dd.n, &rd[t * 4], &ed);
+            double e = 0;
+            dihedral(P3(dd.a0), P3(dd.a1), P3(dd.a2), P3(dd.a3), dd.p0, dd.k, dd.n, &rd[t * 4], &e);
+            count(ed, slot_d, t, e);
         }
     }
     sync();
@@ -401,8 +414,8 @@ LIMA_DEV void local_role(const StepArgs& a, int c, char* lds) {
     if (a.log_rep == r && c == rp.comp_begin) {
         float* o = a.log_data + (size_t)(a.step_count[r] % a.log_ring) * 10;
         const bool by_dihedral = a.enable_dihedrals && nd > 0;
-        if (by_dihedral && p == 0) o[2] = (float)ed;
-        if (!by_dihedral && p == (WAVE ? 0 : P)) o[2] = (float)(eb + ea);
+        if (by_dihedral && p == 0) o[2] = (float)slot_d;
+        if (!by_dihedral && p == (WAVE ? 0 : P)) o[2] = (float)(slot_b + slot_a);
     }
     if (ENERGY) {
         double* e = a.energy + r * kEnergyTerms;
