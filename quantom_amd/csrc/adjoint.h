@@ -361,9 +361,11 @@ LIMA_DEV void adj_solvent_role(const AdjArgs& A, int blk, char* lds) {
 // Chain side of the same sites.  Block = (compound, slice of solv_slice solvents): the transpose
 // of "solvent <- j" with the solvent imaged against the compound's particle 0 and j's stored
 // position, as the forward pass pairs them, and "j <- solvent" for the solvents that the compound
-// lists.  A thread's pairs are all of one pair of types, so it sums dA and dB of 24 eps = 1 over
-// both sites, and the arithmetic site's derivative by 24 eps alone; the geometric one's, times
-// 24 eps, is what is left.  The credits go to both types.
+// lists.  A thread's pairs are all of one pair of types, so it sums each site's derivative by its
+// own 24 eps, and dB of 24 eps = 1 over both sites; dA follows from the three.  The geometric
+// derivative is later divided by 2 eps, so it has a sum of its own: as what the arithmetic one left
+// of both sites' it carried that one's rounding (1,219 solvents, eps_t = eps_0 / 1000: the gradient
+// by eps_t was 4.1e-5 off, 3.1e-6 now).  The credits go to both types.
 // ---------------------------------------------------------------------------
 LIMA_DEV void adj_chain_role(const AdjArgs& A, int blk, double* bins, char* lds) {
     const StepArgs& a = A.s;
@@ -388,7 +390,7 @@ LIMA_DEV void adj_chain_role(const AdjArgs& A, int blk, double* bins, char* lds)
     const float gh = 0.5f * A.gE[r], ga = gh * pa.y, gg = gh * pg.y;
     const float3 wg = make_float3(pg.y * w.x, pg.y * w.y, pg.y * w.z);
     D3 acc{0.0, 0.0, 0.0};
-    double dAs = 0.0, dBs = 0.0, dEa = 0.0;
+    double dBs = 0.0, dEa = 0.0, dEg = 0.0;
     const int s0 = rp.solv_begin + y * A.solv_slice;
     const int s1 = min(s0 + A.solv_slice, rp.solv_end);
     for (int t0 = s0; t0 < s1; t0 += kAdjRows) {
@@ -407,19 +409,19 @@ LIMA_DEV void adj_chain_role(const AdjArgs& A, int blk, double* bins, char* lds)
         // the sites of row j at distance d: the arithmetic one of weight `arith` (0 or 1), the geometric one of `on`
         auto sites = [&](float3 d, float3 v, float arith, float on) {
             const Powers p = powers(d);
-            const float vd = dot3(v, d), ea = arith * pa.y;
+            const float vd = dot3(v, d), wd = dot3(w, d), ea = arith * pa.y;
             const float3 u = make_float3(__builtin_fmaf(ea, v.x, on * wg.x), __builtin_fmaf(ea, v.y, on * wg.y),
                                          __builtin_fmaf(ea, v.z, on * wg.z));
-            const float ud = dot3(u, d), gU = __builtin_fmaf(on, gg, arith * ga);
-            float phi, psi, dA, dB;
+            const float ud = __builtin_fmaf(ea, vd, on * pg.y * wd), gU = __builtin_fmaf(on, gg, arith * ga);
+            float phi, psi;
             phi_psi(p, ab.x, ab.y, phi, psi);
             const float c = __builtin_fmaf(gU, phi, -2.f * ud * psi);
             gather(acc, __builtin_fmaf(phi, u.x, c * d.x), __builtin_fmaf(phi, u.y, c * d.y), __builtin_fmaf(phi, u.z, c * d.z));
-            pair_dab(p, ud, gU, dA, dB);
-            dAs += (double)dA;
-            dBs += (double)dB;
-            // vd phi + g/2 U of 24 eps = 1
-            dEa += (double)(arith * __builtin_fmaf(vd, phi, gh * (-1.f / 6.f) * p.i3 * __builtin_fmaf(0.5f * ab.y, p.i3, ab.x)));
+            dBs += (double)(p.i6 * __builtin_fmaf(ud, p.inv, gU * (-1.f / 12.f)));
+            // of 24 eps = 1: (receiver's weight . d) phi + g/2 U
+            const float energy = gh * (-1.f / 6.f) * p.i3 * __builtin_fmaf(0.5f * ab.y, p.i3, ab.x);
+            dEa += (double)(arith * __builtin_fmaf(vd, phi, energy));
+            dEg += (double)(on * __builtin_fmaf(wd, phi, energy));
         };
         if (!moved) {
 #pragma unroll 2
@@ -436,15 +438,15 @@ LIMA_DEV void adj_chain_role(const AdjArgs& A, int blk, double* bins, char* lds)
             }
         }
     }
-    double v[6] = {acc.x, acc.y, acc.z, dAs, dBs, dEa};
+    double v[6] = {acc.x, acc.y, acc.z, dBs, dEa, dEg};
     group_reduce(t, reinterpret_cast<double*>(lds), v);
     if (t.group == 0 && t.active) {
         A.gxc[(size_t)(kAdjChainSlots + y) * A.n_chain + gi] = make_float4((float)v[0], (float)v[1], (float)v[2], 0.f);
-        double ds, both;
-        chain_rule(v[3], v[4], pa, 1.0, ds, both);
-        const double deg = both - (double)pa.y * v[5];
-        bins_credit(bins, tp, ds, v[5], deg);
-        bins_credit(bins, 0, ds, v[5], deg);
+        // both sites' sum s6 (dA - 2 s6 dB) of 24 eps = 1 gives dA for the chain rule to sigma
+        const double s2 = pa.x, v6 = v[3] * s2 * s2 * s2, eg = pg.y * v[5], both = pa.y * v[4] + eg;
+        const double ds = s2 > 0.0 ? 3.0 * (double)pa.w / s2 * (both - 2.0 * s2 * s2 * s2 * v6) : 0.0;
+        bins_credit(bins, tp, ds, v[4], eg);
+        bins_credit(bins, 0, ds, v[4], eg);
     }
     bins_flush(bins, A.gpar + (size_t)r * kAdjStride);
 }
