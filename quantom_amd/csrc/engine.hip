@@ -470,6 +470,7 @@ struct lima_engine {
     // item: 2 compounds of 128 and 3,000 solvents 22.1 and 9.3, the demo 15.5 and 12.4, 36 compounds
     // of 75 and 11,800 solvents 30 and 23), where every system's items are split.
     static constexpr size_t kListedWideItems = 4096;
+    static constexpr size_t kListedNeighbors = 256, kListedSolvents = 16384;   // the capacities that callers start from (RunParams)
     bool listed_wide() const { return listed_form() == 0 && listed_split_all && max_items <= kListedWideItems; }
     // blocks of the listed compound role: a wavefront per item up to 16,384 wavefronts, which then take several
     int listed_blocks() const {
@@ -1057,13 +1058,17 @@ void validate_and_build(lima_engine* E, const lima_system* sys, int nsys) {
     E->listed_split_all = true;
     for (ReplicaInfo& ri : E->reps_h) {
         const size_t nc = ri.comp_end - ri.comp_begin, nsr = P.enable_solvents ? ri.solv_end - ri.solv_begin : 0;
-        const size_t items = nc == 0 ? 0 : nc * (std::min<size_t>(P.max_compound_neighbors, nc - 1) +
-                                                 (std::min<size_t>(P.max_compound_solvents, nsr) + kSolventChunk - 1) / kSolventChunk);
+        // the most items that lists of these capacities can hold
+        auto items = [&](size_t neighbors, size_t solvents) -> size_t {
+            return nc == 0 ? 0 : nc * (std::min(neighbors, nc - 1) + (std::min(solvents, nsr) + kSolventChunk - 1) / kSolventChunk);
+        };
         int largest = 0;
         for (int c = ri.comp_begin; c < ri.comp_end; c++) largest = std::max(largest, E->comp_off_h[c + 1] - E->comp_off_h[c]);
-        ri.listed_split = items <= lima_engine::kListedWideItems && largest > 32 ? 1 : 0;
+        // The parts group FP32 sums, so whether a system has them follows from the system alone: its items
+        // are counted at the default capacities, and other capacities change no bit of a trajectory.
+        ri.listed_split = items(lima_engine::kListedNeighbors, lima_engine::kListedSolvents) <= lima_engine::kListedWideItems && largest > 32 ? 1 : 0;
         E->listed_split_all = E->listed_split_all && (nc == 0 || ri.listed_split);
-        E->max_items += items;
+        E->max_items += items(P.max_compound_neighbors, P.max_compound_solvents);
     }
 
     // ---- upload ----
