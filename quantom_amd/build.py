@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "liblima_hip.so")
 SOURCES = [os.path.join(HERE, "csrc", "engine.hip")]
-HEADERS = [os.path.join(HERE, "csrc", h) for h in ("device_common.h", "bonded.h", "kernels.h")] + [
+HEADERS = [os.path.join(HERE, "csrc", h) for h in ("device_buffer.h", "device_common.h", "bonded.h", "kernels.h", "adjoint.h")] + [
     os.path.join(ROOT, "include", "lima.h")]
 
 INGEST_LIB = os.path.join(HERE, "liblima_ingest.so")

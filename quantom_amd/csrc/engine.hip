@@ -23,6 +23,7 @@
 
 #include "../../include/lima.h"
 #include "adjoint.h"
+#include "device_buffer.h"
 #include "kernels.h"
 
 using namespace lima;
@@ -37,46 +38,6 @@ constexpr size_t kObservedScratchBytes = (size_t)4 << 20;
 static __device__ __align__(256) unsigned char scratch[kObservedScratchBytes];
 
 namespace {
-
-#define HIP_TRY(expr)                                                                         \
-    do {                                                                                      \
-        hipError_t e_ = (expr);                                                               \
-        if (e_ != hipSuccess) {                                                               \
-            throw LimaError(LIMA_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));   \
-        }                                                                                     \
-    } while (0)
-
-struct LimaError {
-    int code;
-    std::string msg;
-    LimaError(int c, std::string m) : code(c), msg(std::move(m)) {}
-};
-
-template <typename T> struct DBuf {
-    T* p = nullptr;
-    size_t n = 0;
-    DBuf() = default;
-    DBuf(const DBuf&) = delete;
-    DBuf& operator=(const DBuf&) = delete;
-    ~DBuf() { free(); }
-    void alloc(size_t count) {
-        free();
-        n = count;
-        if (count) HIP_TRY(hipMalloc(&p, count * sizeof(T)));
-    }
-    void upload(const std::vector<T>& v) {
-        alloc(std::max<size_t>(v.size(), 1));
-        if (!v.empty()) HIP_TRY(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-    }
-    void zero() {
-        if (p) HIP_TRY(hipMemset(p, 0, n * sizeof(T)));
-    }
-    void free() {
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        n = 0;
-    }
-};
 
 constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mu;
@@ -408,14 +369,15 @@ struct lima_engine {
     }
 
     // Work list of the all-pairs role: per replica, solvent tiles of 256 x chunks of consecutive
-    // compounds; heaviest items first.  Sizes the partial buffer and the LDS tile.
+    // compounds; heaviest items first.  Sizes the partial buffer and the LDS tile.  If there is no
+    // memory for it, the engine keeps the list that it had.
     void build_scwork() {
         const int tile_sz = kStepThreads;
-        scwork_h.clear();
-        kmax = 0;
-        chunk_cap = kRowPad;
+        std::vector<SCWork> work;
+        std::vector<int> counts(R);
+        int most = 0, cap = kRowPad;
         for (int r = 0; r < R; r++) {
-            ReplicaInfo& ri = reps_h[r];
+            const ReplicaInfo& ri = reps_h[r];
             const int target = chunk_target(ri);
             std::vector<std::pair<int, int>> chunks;
             int c = ri.comp_begin;
@@ -427,31 +389,33 @@ struct lima_engine {
                     np += n;
                     c1++;
                 }
-                chunk_cap = std::max(chunk_cap, np);
+                cap = std::max(cap, np);
                 chunks.push_back({c, c1});
                 c = c1;
             }
             if (ri.solv_end == ri.solv_begin) chunks.clear();
-            ri.chunk_count = (int)chunks.size();
-            kmax = std::max(kmax, ri.chunk_count);
+            counts[r] = (int)chunks.size();
+            most = std::max(most, counts[r]);
             for (int t0 = ri.solv_begin; t0 < ri.solv_end; t0 += tile_sz)
                 for (int k = 0; k < (int)chunks.size(); k++)
-                    scwork_h.push_back(SCWork{r, t0, std::min(t0 + tile_sz, ri.solv_end), chunks[k].first, chunks[k].second, k, 0, 0});
+                    work.push_back(SCWork{r, t0, std::min(t0 + tile_sz, ri.solv_end), chunks[k].first, chunks[k].second, k, 0, 0});
         }
-        std::stable_sort(scwork_h.begin(), scwork_h.end(), [&](const SCWork& x, const SCWork& y) {
+        std::stable_sort(work.begin(), work.end(), [&](const SCWork& x, const SCWork& y) {
             const long long wx = (long long)(x.solv_end - x.solv_begin) * (comp_off_h[x.comp_end] - comp_off_h[x.comp_begin]);
             const long long wy = (long long)(y.solv_end - y.solv_begin) * (comp_off_h[y.comp_end] - comp_off_h[y.comp_begin]);
             return wx > wy;
         });
-        const size_t need = std::max<size_t>(1, (size_t)kmax * std::max(NS, 1));
-        if (params.accumulation == LIMA_ACCUM_FIXED64) {
-            if (partS_fx.n < need) partS_fx.alloc(need);
-            if (!partS.p) partS.alloc(1);
-        } else {
-            if (partS.n < need) partS.alloc(need);
-            if (!partS_fx.p) partS_fx.alloc(1);
-        }
-        scwork.upload(scwork_h);
+        const size_t need = std::max<size_t>(1, (size_t)most * std::max(NS, 1));
+        const bool fixed = params.accumulation == LIMA_ACCUM_FIXED64;
+        drop_graphs();   // captured launches name the buffers' addresses
+        partS_fx.grow(fixed ? need : 1);
+        partS.grow(fixed ? 1 : need);
+        scwork.grow(std::max<size_t>(work.size(), 1));
+        if (!work.empty()) HIP_TRY(hipMemcpy(scwork.p, work.data(), work.size() * sizeof(SCWork), hipMemcpyHostToDevice));
+        scwork_h.swap(work);
+        kmax = most;
+        chunk_cap = cap;
+        for (int r = 0; r < R; r++) reps_h[r].chunk_count = counts[r];
     }
 
     // particles per lane of the packed listed role (compounds of at most 16, 32, 64 particles), 0: plain only
@@ -526,6 +490,8 @@ struct lima_engine {
         const ForceBlocks f = force_blocks(roles);
         const int n = f.listed_solvents + xcd_grid(f.thermostat + f.local + f.bridges + f.all_pairs + f.listed);
         if (n == 0) return;
+        if (f.all_pairs && ((FIXED ? partS_fx.n : partS.n) < (size_t)kmax * NS || scwork.n < scwork_h.size()))
+            throw LimaError(LIMA_E_HIP, "the all-pairs work list has no device memory");
         const int ppl = listed_form() == 1 ? pack_ppl() : 0;
         const size_t lds = force_lds(f, ppl);
         switch (ppl) {
@@ -1243,9 +1209,7 @@ void load_state(lima_engine* E, const float4* src) {
     d2d(E->sprev.p, src + 2 * nch + ns, ns * 16, E->stream);
 }
 
-template <typename T> void ensure(DBuf<T>& b, size_t n) {
-    if (b.n < n) b.alloc(n);
-}
+template <typename T> void ensure(DBuf<T>& b, size_t n) { b.grow(n); }
 
 // per-particle constants of the adjoint (once per engine)
 void adj_setup(lima_engine* E) {
@@ -1890,7 +1854,7 @@ int io_layout(lima_engine* E, const IoArray (&io)[4], IoArrays& a) {
         a.p[k] = io[k].dev;
         a.end[k] = (int)(total += io[k].host ? io[k].n : 0);
     }
-    if (total && E->io_dev.n < 3 * total) E->io_dev.alloc(3 * total);
+    E->io_dev.grow(3 * total);
     if (total && total * 12 <= kIoPinned && !E->io_pinned) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&E->io_pinned), kIoPinned, 0));
     return (int)total;
 }
@@ -2162,8 +2126,8 @@ int lima_step_logged(lima_engine* E, int32_t n, int32_t system, int32_t slots, f
         HIP_TRY(hipSetDevice(E->device));
         HIP_TRY(hipStreamSynchronize(E->stream));
         const size_t per_step = (size_t)nc * std::max(slots, 1) * 9;
-        if (E->log_data.n < (size_t)kLogRing * 10) E->log_data.alloc((size_t)kLogRing * 10);
-        if (traindata && E->train_data.n < kLogRing * per_step) E->train_data.alloc(kLogRing * per_step);
+        E->log_data.grow((size_t)kLogRing * 10);
+        if (traindata) E->train_data.grow(kLogRing * per_step);
         // the rings enter the captured step through its arguments: recapture with them, and again without
         auto reset_graph = [&] {
             E->drop_graphs();
