@@ -176,7 +176,9 @@ struct lima_engine {
     DBuf<float4> ss_part, ss_img;
     DBuf<float> comp_cs_bound;
     AdjBufs adjb;
-    DBuf<float> io_dev;           // triples of the state or forces on their way (io_get, io_set)
+    // triples of the state or forces on their way (io_get, io_set): of four arrays, allocated with the
+    // engine, so that its state can be read whatever has become of the device's memory since
+    DBuf<float> io_dev;
     float* io_pinned = nullptr;
     uint32_t* err_pinned = nullptr;   // the error words as of the last fetch_errors
 
@@ -1134,6 +1136,7 @@ void validate_and_build(lima_engine* E, const lima_system* sys, int nsys) {
     E->cell_ids.alloc(NSx); E->solv_cell.alloc(NSx);
     E->cell_rep.upload(cell_rep_h);
     E->comp_cs_bound.upload(cs_bound);
+    E->io_dev.alloc((size_t)6 * std::max(E->NCH + E->NS, 1));
     E->ss_part.alloc(NSx); E->ss_part.zero();
     E->ss_img.alloc(NSx); E->ss_img.zero();
 }
@@ -1854,7 +1857,6 @@ int io_layout(lima_engine* E, const IoArray (&io)[4], IoArrays& a) {
         a.p[k] = io[k].dev;
         a.end[k] = (int)(total += io[k].host ? io[k].n : 0);
     }
-    E->io_dev.grow(3 * total);
     if (total && total * 12 <= kIoPinned && !E->io_pinned) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&E->io_pinned), kIoPinned, 0));
     return (int)total;
 }

@@ -42,3 +42,30 @@ def test_large_unpinned_forces_equal_the_small_ones(small_system):
         assert np.array_equal(c[r * len(c1):(r + 1) * len(c1)], c1) and np.array_equal(s[r * len(s1):(r + 1) * len(s1)], s1)
     one.close()
     many.close()
+
+
+def test_state_and_forces_take_no_device_memory(small_system):
+    """Reading and setting the state, and forces, work where nothing is left on the device: the first
+    call allocates nothing there."""
+    import ctypes as C
+
+    from quantom_amd.abi import RunParams
+    from quantom_amd.engine import Engine, load_library
+    load_library()
+    hip = C.CDLL("libamdhip64.so.7")        # the runtime that the library has loaded
+
+    def free():
+        n, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(n), C.byref(total)) == 0
+        return n.value
+
+    e = Engine([small_system] * 120, RunParams(nlist_interval=0))
+    e.compute_forces()                      # code and pinned buffers loaded
+    f = Engine([small_system] * 120, RunParams(nlist_interval=0))
+    before = free()
+    state = f.get_state()
+    f.set_state(*state)
+    f.compute_forces()
+    assert free() == before
+    e.close()
+    f.close()
