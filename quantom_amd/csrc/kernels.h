@@ -470,6 +470,7 @@ LIMA_DEV void replay_images(const StepArgs& a, int cb, int ce, float4* p0s, floa
 // issue time, one reciprocal shared by two or four pairs saves 1-2% and loses accuracy.
 // ---------------------------------------------------------------------------
 constexpr int kRowPad = 4;
+constexpr float kFarAway = 1e18f;   // outside any box; r^2 = 3e36 is finite, its reciprocal's square is zero
 constexpr int kAllPairsHead = 528;   // the constants and row offsets before the tile, 16-byte aligned
 static_assert(kMaxTypes * 8 + (kChunkCompounds + 1) * 4 <= kAllPairsHead && kAllPairsHead % 16 == 0, "head of the tile");
 inline size_t all_pairs_lds_bytes(int rows) {
@@ -520,7 +521,7 @@ template <bool FIXED, bool ENERGY> LIMA_DEV void all_pairs_role(const StepArgs& 
     }
     for (int k = tid; k < total; k += kStepThreads) {
         const int src = a.row_src[base + k];
-        float4 p = make_float4(1e3f, 1e3f, 1e3f, 0.f);   // padding: a finite distance, zero constants
+        float4 p = make_float4(kFarAway, kFarAway, kFarAway, 0.f);   // padding: zero constants, at a distance that is not zero
         float2 ab = make_float2(0.f, 0.f);
         if (src >= 0) {
             p = a.cpos[src];
@@ -596,7 +597,6 @@ constexpr int kListedParts = 4;
 // rows of a part of an item of `nsrc` sources: a quarter, in whole fours, or all of them
 LIMA_DEV int listed_part(int nsrc, int split) { return nsrc <= 32 || !split ? (nsrc + 3) & ~3 : ((nsrc + 15) >> 4) * 4; }
 
-constexpr float kFarAway = 1e18f;   // r^2 = 3e36 is finite, its reciprocal's square is zero
 constexpr size_t kListedLds = (size_t)kMaxTypes * kMaxTypes * sizeof(float2) + 4 * kSolventChunk * sizeof(float4);
 static_assert(kListedParts == kStepThreads / 64 && kSolventChunk + kListedParts * kCompoundBlock <= 4 * kSolventChunk,
               "a wavefront per part; the rows and the parts' sums of the wide form");
