@@ -69,9 +69,10 @@ LIMA_DEV float fmul(float a, float b) {
     return a * b;
 }
 
-// Float3::len (QuantomTypes.cuh:60): sqrtf((x*x + y*y) + z*z), correctly rounded
+// Float3::len (QuantomTypes.cuh:60): sqrtf((x*x + y*y) + z*z), correctly rounded: sqrtf is, as the
+// library is compiled, while HIP's __fsqrt_rn is the hardware root and up to an ulp off
 LIMA_DEV float exact_len(float x, float y, float z) {
-    return __fsqrt_rn(fadd(fadd(fmul(x, x), fmul(y, y)), fmul(z, z)));
+    return sqrtf(fadd(fadd(fmul(x, x), fmul(y, y)), fmul(z, z)));
 }
 
 // The box of a system, in vector registers.  A wave64 FP32 add, multiply or FMA whose operands

@@ -64,3 +64,21 @@ def test_potential_slot_is_thread_0s_terms(kind, csize, times):
     extra = _energy(s, kind, 64) if n > 64 else 0.0
     assert n <= 64 or abs(extra) > 1e-3 * abs(want)     # a sum with term 64 would be seen
     assert abs(log[0, 2] - want) <= 1e-4 * abs(want), (log[0, 2], want, extra)
+
+
+def test_force_magnitude_is_correctly_rounded(small_system):
+    """|F| of the log (Float3::len) is the correctly rounded root of the FP32 sum of squares, as the
+    reference's sqrtf and the oracle's are: bit for bit over 64 steps."""
+    from quantom_amd.engine import Engine
+    p = RunParams(nlist_interval=10)
+    a, b = Engine([small_system], p), Engine([small_system], p)
+    log, _ = a.step_logged(64, 0, 128, train=False)
+    want = []
+    for _ in range(64):
+        b.step(1)
+        f = b.forces()[0][0]
+        q = f * f                                        # float32, each operation rounded
+        want.append(np.sqrt((q[0] + q[1]) + q[2]))
+    a.close()
+    b.close()
+    assert np.array_equal(log[:, 3], np.array(want, np.float32))
