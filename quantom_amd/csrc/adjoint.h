@@ -207,7 +207,8 @@ struct AdjArgs {
     int nb, na;              // most bonds and angles of any compound (LDS strides)
 };
 struct AdjBlocks {
-    int bonded, bridges, intra, listed, solvent, chain, pairs;   // blocks of each role, in this order
+    int bonded, bridges, intra, listed, solvent, chain, pairs;   // blocks of each role
+    int width;                                                   // the grid's (grid_of)
 };
 constexpr int kAdjThreads = 256;
 constexpr int kAdjChainSlots = 3;
@@ -801,7 +802,7 @@ __global__ __launch_bounds__(kAdjThreads, 4) void adj_frame_kernel(AdjArgs A, Ad
     extern __shared__ float4 dyn_lds[];
     double* bins = reinterpret_cast<double*>(dyn_lds);
     char* lds = reinterpret_cast<char*>(dyn_lds) + kAdjHead;
-    int b = blockIdx.x;
+    int b = blockIdx.y * f.width + blockIdx.x;
     if (b < f.bridges) {
         const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         adj_bridge_role(A, 4 * b + wid, reinterpret_cast<AdjBridgeStage*>(lds)[wid]);

@@ -489,18 +489,20 @@ struct lima_engine {
     }
 
     template <bool FIXED, bool ENERGY> void launch_roles(const StepArgs& a, int roles) {
-        const ForceBlocks f = force_blocks(roles);
+        ForceBlocks f = force_blocks(roles);
         const int n = f.listed_solvents + xcd_grid(f.thermostat + f.local + f.bridges + f.all_pairs + f.listed);
         if (n == 0) return;
         if (f.all_pairs && ((FIXED ? partS_fx.n : partS.n) < (size_t)kmax * NS || scwork.n < scwork_h.size()))
             throw LimaError(LIMA_E_HIP, "the all-pairs work list has no device memory");
         const int ppl = listed_form() == 1 ? pack_ppl() : 0;
         const size_t lds = force_lds(f, ppl);
+        const dim3 grid = grid_of(n);
+        f.width = (int)grid.x;
         switch (ppl) {
-            case 1: step_forces_kernel<FIXED, ENERGY, 1><<<n, kStepThreads, lds, stream>>>(a, f); break;
-            case 2: step_forces_kernel<FIXED, ENERGY, 2><<<n, kStepThreads, lds, stream>>>(a, f); break;
-            case 4: step_forces_kernel<FIXED, ENERGY, 4><<<n, kStepThreads, lds, stream>>>(a, f); break;
-            default: step_forces_kernel<FIXED, ENERGY, 0><<<n, kStepThreads, lds, stream>>>(a, f);
+            case 1: step_forces_kernel<FIXED, ENERGY, 1><<<grid, kStepThreads, lds, stream>>>(a, f); break;
+            case 2: step_forces_kernel<FIXED, ENERGY, 2><<<grid, kStepThreads, lds, stream>>>(a, f); break;
+            case 4: step_forces_kernel<FIXED, ENERGY, 4><<<grid, kStepThreads, lds, stream>>>(a, f); break;
+            default: step_forces_kernel<FIXED, ENERGY, 0><<<grid, kStepThreads, lds, stream>>>(a, f);
         }
     }
     template <bool ADVANCE, bool FIXED, bool ENERGY> void launch_integrate(const StepArgs& a, bool compounds, bool solvents) {
@@ -546,7 +548,7 @@ struct lima_engine {
         const bool solv = params.enable_solvents && NS > 0;
         if (NC > 0) nl_compound_compound_kernel<<<NC, 64, 0, stream>>>(a);
         if (solv) {
-            const int blocks = NC * max_segs + (NS + 255) / 256;
+            const dim3 blocks = grid_of((long long)NC * max_segs + (NS + 255) / 256);
             nl_count_kernel<<<blocks, 256, 0, stream>>>(a);
             nl_cell_scan_kernel<<<1, 1024, 0, stream>>>(a);
             nl_write_kernel<<<blocks, 256, 0, stream>>>(a);
@@ -1373,7 +1375,9 @@ void adj_frame(lima_engine* E, int j, const float4* X, const float4* rs_prev, co
                                             sizeof(AdjPairStage), 4 * sizeof(AdjBridgeStage),
                                             adj_bonded_lds(E->max_cb, E->max_ca, E->max_cd)});
     const int blocks = f.bonded + f.bridges + f.intra + f.listed + f.chain + f.pairs + f.solvent;
-    if (blocks > 0) adj_frame_kernel<<<blocks, kAdjThreads, lds, E->stream>>>(A, f);
+    const dim3 grid = grid_of(blocks);
+    f.width = (int)grid.x;
+    if (blocks > 0) adj_frame_kernel<<<grid, kAdjThreads, lds, E->stream>>>(A, f);
     adj_update_kernel<<<(N + 255) / 256, 256, 0, E->stream>>>(A, kAdjChainSlots + (sv ? B.n_sslices : 0), sv ? B.n_cchunks + 1 : 0,
                                                               a1, a2, a_out, rs_prev, B.cfac.p, B.w.p);
 }

@@ -18,6 +18,7 @@
 // box length, time step and type tables of that replica, so one launch covers
 // any number of independent systems.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 #include "bonded.h"
 #include "device_common.h"
@@ -155,6 +156,16 @@ __host__ LIMA_DEV float4 solvent_pos(float x, float y, float z, float L) {
 // never meet a block barrier.
 // ===========================================================================
 constexpr int kStepThreads = 256;
+
+// A launch of 2^32 threads or more in one dimension is refused (2^24 blocks of 256), which an all-pairs
+// list of a million solvents and as many particles, or its list build, reaches: blocks beyond kGridWidth
+// take a second dimension.  Whole rows, so the last one's rest have no work; widths are multiples of 8,
+// which keeps a block's XCD that of its number.
+constexpr long long kGridWidth = 1 << 14;
+inline dim3 grid_of(long long blocks) {
+    const long long rows = std::max<long long>(1, (blocks + kGridWidth - 1) / kGridWidth);
+    return dim3(rows == 1 ? (unsigned)blocks : (unsigned)(((blocks + rows - 1) / rows + 7) / 8 * 8), (unsigned)rows);
+}
 
 LIMA_DEV void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1392,6 +1403,7 @@ struct ForceBlocks {
     int listed_wide;      // 1: a block per listed item
     int spread;           // groups of eight other blocks after each group of eight solvent-list blocks
     int mix;              // all-pairs blocks after each listed block; 0: all of them first
+    int width;            // the grid's (grid_of)
 };
 
 template <bool FIXED, bool ENERGY, int PPL>
@@ -1399,14 +1411,15 @@ __global__ __launch_bounds__(kStepThreads, ENERGY ? 2 : 4) void step_forces_kern
     extern __shared__ float4 dyn_lds[];
     char* lds = reinterpret_cast<char*>(dyn_lds);
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int unit = blockIdx.x / kXcds, turn = unit / (f.spread + 1), lists = f.listed_solvents / kXcds;
+    const int block = blockIdx.y * f.width + blockIdx.x;
+    const int unit = block / kXcds, turn = unit / (f.spread + 1), lists = f.listed_solvents / kXcds;
     if (turn < lists && unit % (f.spread + 1) == 0) {
-        const int item = xcd_item(turn * kXcds + blockIdx.x % kXcds, f.listed_solvents);
+        const int item = xcd_item(turn * kXcds + block % kXcds, f.listed_solvents);
         if (item >= f.solvent_items) return;
         solvent_listed_role<ENERGY>(a, item, f.solvent_rounds);
         return;
     }
-    int b = blockIdx.x - min(turn + 1, lists) * kXcds;   // among the other roles' blocks
+    int b = block - min(turn + 1, lists) * kXcds;   // among the other roles' blocks
     // Between the steps of a captured graph the thermostat of one runs beside the forces of the
     // next, which do not read what it writes (lambda, the counters): its own launch took 3.9 us of
     // a small system's 31 us step.
@@ -1442,7 +1455,7 @@ __global__ __launch_bounds__(kStepThreads, ENERGY ? 2 : 4) void step_forces_kern
         all_pairs_role<FIXED, ENERGY>(a, all_pairs, lds);
         return;
     }
-    if (listed >= f.listed) return;   // the launch is padded to whole groups of eight
+    if (listed >= f.listed) return;   // the launch is padded to whole groups of eight, and to whole rows
     if constexpr (PPL == 0) {
         if (f.listed_wide) listed_role<FIXED, ENERGY, true>(a, listed, f.listed, lds);
         else listed_role<FIXED, ENERGY, false>(a, listed, f.listed, lds);
@@ -2022,14 +2035,14 @@ LIMA_DEV void nl_cell_scatter(const NlistArgs& a, int block) {
 // is its launches, about 5 us each: eleven took 54 us, seven (the counters cleared by the sort, few
 // compounds' items written by the work list's block) save 10 to 13 of a rebuild.
 __global__ __launch_bounds__(256) void nl_count_kernel(NlistArgs a) {
-    const int b = blockIdx.x, cs = a.n_comp * a.max_segs;
-    if (b < cs) nl_cs_count(a, b % a.n_comp, b / a.n_comp);
-    else nl_cell_count(a, b - cs);
+    const long long b = (long long)blockIdx.y * gridDim.x + blockIdx.x, cs = (long long)a.n_comp * a.max_segs;
+    if (b < cs) nl_cs_count(a, (int)(b % a.n_comp), (int)(b / a.n_comp));
+    else nl_cell_count(a, (int)(b - cs));
 }
 __global__ __launch_bounds__(256) void nl_write_kernel(NlistArgs a) {
-    const int b = blockIdx.x, cs = a.n_comp * a.max_segs;
-    if (b < cs) nl_cs_write(a, b % a.n_comp, b / a.n_comp);
-    else nl_cell_scatter(a, b - cs);
+    const long long b = (long long)blockIdx.y * gridDim.x + blockIdx.x, cs = (long long)a.n_comp * a.max_segs;
+    if (b < cs) nl_cs_write(a, (int)(b % a.n_comp), (int)(b / a.n_comp));
+    else nl_cell_scatter(a, (int)(b - cs));
 }
 
 // sort each cell's ids ascending (rank sort in LDS), making the lists deterministic, and clear its
