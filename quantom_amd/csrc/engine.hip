@@ -552,8 +552,8 @@ struct lima_engine {
             nl_count_kernel<<<blocks, 256, 0, stream>>>(a);
             nl_cell_scan_kernel<<<1, 1024, 0, stream>>>(a);
             nl_write_kernel<<<blocks, 256, 0, stream>>>(a);
-            nl_cell_sort_kernel<<<n_cells, 256, 0, stream>>>(a);
-            nl_solvent_solvent_kernel<<<xcd_grid(n_cells), kSolventListThreads, 0, stream>>>(a);
+            nl_cell_sort_kernel<<<grid_of(n_cells), 256, 0, stream>>>(a);
+            nl_solvent_solvent_kernel<<<grid_of(xcd_grid(n_cells)), kSolventListThreads, 0, stream>>>(a);
         }
         launch_work_list(a, stream);
     }

@@ -2050,7 +2050,8 @@ __global__ __launch_bounds__(256) void nl_write_kernel(NlistArgs a) {
 __global__ __launch_bounds__(256) void nl_cell_sort_kernel(NlistArgs a) {
     constexpr int CAP = 2048;
     __shared__ int ids[CAP];
-    const int cell = blockIdx.x;
+    const int cell = blockIdx.y * gridDim.x + blockIdx.x;
+    if (cell >= a.n_cells) return;
     if (threadIdx.x == 0) a.cell_cnt[cell] = 0;
     const int b = a.cell_start[cell], n = a.cell_start[cell + 1] - b;
     if (n > CAP) {
@@ -2095,7 +2096,7 @@ __global__ __launch_bounds__(kSolventListThreads) void nl_solvent_solvent_kernel
     __shared__ unsigned short queue[kSolventListThreads / 64][kSsQueue];
     __shared__ int cell_b[27], cell_n[27], cell_off[28];
     // cells of one replica are contiguous: XCD-contiguous order keeps a replica's positions in one L2
-    const int cell = xcd_item(blockIdx.x, gridDim.x);
+    const int cell = xcd_item(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     if (cell >= a.n_cells) return;
     const int h0 = a.cell_start[cell], h1 = a.cell_start[cell + 1];
     if (h0 == h1) return;

@@ -34,3 +34,28 @@ def test_list_build_over_2_to_the_24_blocks():
         assert np.array_equal(got[2][s], want_ss[s]), s
     for e in (both, one, other):
         e.close()
+
+
+@pytest.mark.parametrize("box,cells", [(200.0, 166 ** 3), (310.0, 256 ** 3)])
+def test_list_build_over_many_cells(box, cells):
+    """Boxes of 4.6 million cells (over 2^32 threads at 1,024 a cell) and of 16.8 million (at 256, whose
+    launch clears the cells' counters for the next build): built twice, the lists are the oracle's."""
+    from oracle.oracle import KIND_CS, KIND_SS, Oracle
+    from quantom_amd.abi import RunParams
+    from quantom_amd.engine import Engine
+    rng = np.random.default_rng(9)
+    g = np.stack(np.meshgrid(*[np.arange(8) * 0.5] * 3, indexing="ij"), -1).reshape(-1, 3)
+    x = np.mod(np.concatenate([g + c for c in ((0.2, 0.2, 0.2), (box - 2.1, 0.3, box / 2), (box / 2,) * 3)])
+               + rng.uniform(-0.05, 0.05, (3 * len(g), 3)), box)
+    s = ms.build(box, [([(3.0, 3.0, 5.0), (3.1, 3.0, 5.0)], [1, 2])], x)
+    p = RunParams(nlist_interval=0)
+    e, o = Engine([s], p), Oracle(s, p, precision=32)
+    assert e.config()["n_cells"] == cells
+    o.compute_forces()
+    for build in range(2):
+        _, cs, ss = e.neighbors()
+        for got, want in ((cs, o.neighbors(KIND_CS)), (ss, o.neighbors(KIND_SS))):
+            assert sum(map(len, want)) > 0
+            assert all(np.array_equal(np.sort(a), np.sort(b)) for a, b in zip(got, want)), build
+        e.rebuild_neighbors()
+    e.close()
