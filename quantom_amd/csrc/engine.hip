@@ -420,6 +420,13 @@ struct lima_engine {
         for (int r = 0; r < R; r++) reps_h[r].chunk_count = counts[r];
     }
 
+    // a failed growth that could not even give the former buffers back
+    void check_work_list() const {
+        const size_t partials = params.accumulation == LIMA_ACCUM_FIXED64 ? partS_fx.n : partS.n;
+        if (partials < (size_t)kmax * NS || scwork.n < scwork_h.size())
+            throw LimaError(LIMA_E_HIP, "the all-pairs work list has no device memory");
+    }
+
     // particles per lane of the packed listed role (compounds of at most 16, 32, 64 particles), 0: plain only
     int pack_ppl() const { return max_cn <= 16 ? 1 : max_cn <= 32 ? 2 : max_cn <= 64 ? 4 : 0; }
 
@@ -492,8 +499,7 @@ struct lima_engine {
         ForceBlocks f = force_blocks(roles);
         const int n = f.listed_solvents + xcd_grid(f.thermostat + f.local + f.bridges + f.all_pairs + f.listed);
         if (n == 0) return;
-        if (f.all_pairs && ((FIXED ? partS_fx.n : partS.n) < (size_t)kmax * NS || scwork.n < scwork_h.size()))
-            throw LimaError(LIMA_E_HIP, "the all-pairs work list has no device memory");
+        if (f.all_pairs) check_work_list();
         const int ppl = listed_form() == 1 ? pack_ppl() : 0;
         const size_t lds = force_lds(f, ppl);
         const dim3 grid = grid_of(n);
@@ -647,6 +653,7 @@ struct lima_engine {
     void ensure_graphs() {
         if (graphs_ready) return;
         drop_graphs();
+        check_work_list();   // not inside a capture
         const int save_cur = cur;
         const long long save_step = step, save_since = since_rebuild, save_nr = n_rebuilds, save_dev = dev_step;
         const int iv = params.nlist_interval;
