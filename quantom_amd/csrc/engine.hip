@@ -1757,7 +1757,6 @@ void set_parameters(lima_engine* E, int r, const double* v) {
     set_parameters_kernel<<<1, kMaxTypes * kMaxTypes, 0, E->stream>>>(sp, r, E->tab_sc.p, E->tab_cs.p, E->tab_ss.p, E->tab_inter.p,
                                                                       E->tab_intra.p, E->tab_inter_ab.p, E->tab_intra_ab.p, E->bonds.p,
                                                                       E->angles.p, E->brb.p, E->bra.p);
-    HIP_TRY(hipGetLastError());
 }
 
 thread_local std::string g_last_error;
