@@ -94,6 +94,10 @@ LIMA_DEV Box make_box(float L, float half) {
 LIMA_DEV float above_half(float t, const Box& box) {
     return __builtin_amdgcn_fmed3f(__builtin_fmaf(t, box.step, box.nstep), 0.f, 1.f);
 }
+// Whether any of three separations is exactly half a box: their two images are equally near.
+LIMA_DEV bool half_a_box(float dx, float dy, float dz, float half) {
+    return (fabsf(dx) == half) | (fabsf(dy) == half) | (fabsf(dz) == half);
+}
 
 // LIMAENG::applyHyperpos (Engine.cuh:24-30) on one coordinate
 // m + L*flag with flag 0 or 1: the product is exact, so one fused operation

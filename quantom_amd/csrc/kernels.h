@@ -471,9 +471,12 @@ LIMA_DEV void replay_images(const StepArgs& a, int cb, int ce, float4* p0s, floa
 // reference carries the image from compound to compound (Engine.cu:1111).  With the solvent and
 // every particle 0 inside the box both are the image nearest to particle 0 (a carried image lies
 // within [-L/2, 3L/2], one shift from it), and the direct one is rounded once instead of once a
-// shift.  Where any of them lies outside (positions as a caller first set them), the sequence is
-// replayed from the first compound.  The replay had cost 7% of the kernel on the production
-// system's 100 compounds and 14% on the 18 nm box's 400.
+// shift.  Where the two are exactly half a box apart both images are as near and the carried one
+// depends on the compounds before: there, and for a whole block where a solvent or a particle 0 lies
+// outside (positions as a caller first set them), the sequence is replayed from the first compound.
+// The replay had cost 7% of the kernel on the production system's 100 compounds and 14% on the 18 nm
+// box's 400; the test for a tie costs the demo's step (compounds of 30 to 43 particles) 1%, larger
+// compounds' less.
 //
 // Bound: VALU issue, 14 instructions a pair at the full rate (2.3 cycles) and a reciprocal (12-16
 // cycles among FMAs): 50 cycles a pair of 64 lanes measured with one solvent a lane, 51-54 with
@@ -550,7 +553,25 @@ template <bool FIXED, bool ENERGY> LIMA_DEV void all_pairs_role(const StepArgs& 
         const float4 q0 = tile[j0];
         float sx = rx, sy = ry, sz = rz, lx = 0.f, ly = 0.f, lz = 0.f;
         hyperpos(q0.x, q0.y, q0.z, sx, sy, sz, box);
-        if (!direct) { rx = sx; ry = sy; rz = sz; }
+        if (!direct) {
+            rx = sx; ry = sy; rz = sz;
+        } else if (__ballot(half_a_box(fsub(q0.x, rx), fsub(q0.y, ry), fsub(q0.z, rz), rp.half)) != 0ull) {
+            // A tie (one or two a step of production's 7 million): the image carried from the last
+            // compound before that ties with none of these solvents, where it is the nearest again.
+            int c = c0 + ci - 1;
+            for (; c >= rp.comp_begin; c--) {
+                const float4 q = a.cpos[a.comp_off[c]];
+                if (__ballot(half_a_box(fsub(q.x, rx), fsub(q.y, ry), fsub(q.z, rz), rp.half)) == 0ull) break;
+            }
+            float cx = rx, cy = ry, cz = rz;
+            for (c = max(c, rp.comp_begin); c <= c0 + ci; c++) {
+                const float4 q = a.cpos[a.comp_off[c]];
+                hyperpos(q.x, q.y, q.z, cx, cy, cz, box);
+            }
+            if (fabsf(fsub(q0.x, rx)) == rp.half) sx = cx;
+            if (fabsf(fsub(q0.y, ry)) == rp.half) sy = cy;
+            if (fabsf(fsub(q0.z, rz)) == rp.half) sz = cz;
+        }
         for (int j = j0; j < j1; j += kRowPad) {
             float4 q[kRowPad];
 #pragma unroll
@@ -1136,7 +1157,8 @@ LIMA_DEV void listed_packed_role(const StepArgs& a, int blk, int nblk, char* lds
 // of the move.  The particle 0s set one if the farthest of them on that side does.  Entries are then
 // independent: a quad of lanes walks a row, lane x of it entries 4x .. 4x + 3 of every 16, and the
 // four sums are added in a fixed order.  Where any position lies outside (a solvent's w, particle 0
-// as a caller first set it) the wavefront replays the sequence, with the same split of the sums.
+// as a caller first set it), or an entry is exactly half a box away, where the sequence keeps the image
+// that it has, the wavefront replays the sequence, with the same split of the sums.
 //
 // Bound by the gathers: an entry takes 24 full-rate instructions and a reciprocal, 70 cycles a
 // wavefront, and 64 lines of L1.  The carried image had taken 32 and made a row one serial chain.
@@ -1199,6 +1221,9 @@ template <bool ENERGY> LIMA_DEV void solvent_listed_role(const StepArgs& a, int 
     const float4 pv = a.tab_ss[r];
     float2 pss = lj_ab(pv.x, pv.y);
     asm("" : "+v"(pss.x), "+v"(pss.y));   // full rate, as the box's
+    // Entries can be half a box away only where that is within the lists' radius and what solvents drift
+    // between builds (a quarter of it); tested for everywhere, they cost the 256 replicas' step 1%.
+    const bool near_ties = rp.half * rp.half < 1.5625f * rp.ss_bound;
     // the particle 0s: inside the box, and the farthest on either side of each axis
     float p0_outside = 0.f;
     const int last = rp.comp_end - 1;
@@ -1240,6 +1265,7 @@ template <bool ENERGY> LIMA_DEV void solvent_listed_role(const StepArgs& a, int 
         };
         float evx = farthest(me.x, 0, sdx), evy = farthest(me.y, 1, sdy), evz = farthest(me.z, 2, sdz);
         float lx = 0.f, ly = 0.f, lz = 0.f;
+        bool tie = false;
         double e_round = 0.0, w_round = 0.0;
         // past the row's count a lane re-reads its entries of the first segment (in bounds, not used)
         // and its own position
@@ -1287,19 +1313,26 @@ template <bool ENERGY> LIMA_DEV void solvent_listed_role(const StepArgs& a, int 
                 };
                 if (__ballot(n < 4) == 0ull) sums(std::true_type{});
                 else sums(std::false_type{});
+                if (near_ties)
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+                        tie = tie | half_a_box(fsub(cur.q[u].x, me.x), fsub(cur.q[u].y, me.y), fsub(cur.q[u].z, me.z), rp.half);
                 cur = nxt;
             }
         }
         float mx = me.x, my = me.y, mz = me.z;
-        if (__ballot(outside != 0.f) == 0ull) {
+        float4 end = me;   // the sequence's last entry
+        if (cnt > 0) end = a.spos[row[cnt - 1]];
+        else if (last >= rp.comp_begin) end = a.cpos[a.comp_off[last]];
+        tie = tie | half_a_box(fsub(end.x, me.x), fsub(end.y, me.y), fsub(end.z, me.z), rp.half);
+        if (__ballot(outside != 0.f || tie) == 0ull) {
             evx = quad_sum(evx);
             evy = quad_sum(evy);
             evz = quad_sum(evz);
             if (cnt > 0 || last >= rp.comp_begin) {
-                const float4 q = cnt > 0 ? a.spos[row[cnt - 1]] : a.cpos[a.comp_off[last]];
-                mx = last_image(me.x, q.x, evx, sdx, box);
-                my = last_image(me.y, q.y, evy, sdy, box);
-                mz = last_image(me.z, q.z, evz, sdz, box);
+                mx = last_image(me.x, end.x, evx, sdx, box);
+                my = last_image(me.y, end.y, evy, sdy, box);
+                mz = last_image(me.z, end.z, evz, sdz, box);
             }
         } else {
             lx = ly = lz = 0.f;
