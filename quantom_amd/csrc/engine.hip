@@ -58,14 +58,15 @@ unsigned char* scratch_address(int device) {
 }
 
 struct LaunchConfig {
-    int spt = 1;                  // solvents per lane of the all-pairs role (reported; always 1)
+    int spt = 1;                  // solvents per lane of the all-pairs role: 1 (a field of saved tunings, and reported)
     int chunk_particles = 0;      // target chain particles per solvent<-chain work item (0: by each system's size)
     int listed_grid = 0;          // wavefront pairs of the listed compound role (0: by the number of items)
     int use_graph = 1;
-    int listed_lanes = 0;         // 1 or 4, as saved by earlier versions and reported; the listed solvent role takes four lanes a solvent
+    int listed_lanes = 4;         // lanes per solvent of the listed solvent role: 4 (saved tunings may say 1: reported, the same role)
     int listed_packed = -1;       // compounds of <= 64 particles: the packed listed role (1), the plain one (0), or
                                   // (FP32) the plain one with small compounds' rows split (2); -1: by the number of compounds
-    int fused_thermostat = 0;     // 0: the thermostat as its own kernel; 1, 2: in the integrate launch's last blocks
+    int fused_thermostat = 0;     // 0: the thermostat as its own kernel; 1: in the integrate launch's last blocks (saved tunings
+                                  // may say 2, a second form when the integrators were two launches: reported, the same)
 };
 
 // Device buffers of lima_adjoint_run / lima_record_frames, grown on demand and
@@ -152,11 +153,8 @@ struct lima_engine {
     DBuf<double> ke_comp, ke_stile, temperature, energy;
     DBuf<long long> step_count;   // per replica: steps done (the reference cadence thermostat reads it)
     DBuf<int> thermo_cnt, thermo_total;   // the thermostat in the integrators' last blocks
-    bool thermo_ok = false;       // every system has integrator blocks for it (form 1)
-    bool thermo_ok_comp = false;  // every system has compounds (form 2)
-    int thermo_form() const {
-        return cfg.fused_thermostat == 1 && thermo_ok ? 1 : cfg.fused_thermostat == 2 && thermo_ok_comp ? 2 : 0;
-    }
+    bool thermo_ok = false;       // every system has integrator blocks for it
+    int thermo_form() const { return thermo_ok ? cfg.fused_thermostat : 0; }
     bool thermo_fused() const { return thermo_form() != 0; }
     // While a graph of several steps is captured: the step being enqueued starts with the thermostat
     // of the one before, and leaves its own to the next.  Not where a force role reads or writes what
@@ -1121,23 +1119,17 @@ void validate_and_build(lima_engine* E, const lima_system* sys, int nsys) {
     E->temperature.alloc(nsys); E->temperature.zero();
     E->step_count.alloc(nsys); E->step_count.zero();
     {
-        // the thermostat runs in the integrators' last block of each system when every system has
-        // integrator blocks of the kind that runs after the all-pairs kernel (its solvent tiles,
-        // when solvents are on: the thermostat of system 0 also closes that kernel's clock span)
+        // the thermostat can run in a system's last integrator block where every system has one
         const bool solv = E->params.enable_solvents && E->NS > 0;
         std::vector<int> total(nsys);
-        bool ok = true, ok_comp = E->NC > 0;
+        E->thermo_ok = true;
         for (int r = 0; r < nsys; r++) {
             const ReplicaInfo& ri = E->reps_h[r];
-            const int tiles = solv ? ri.stile_end - ri.stile_begin : 0;
-            total[r] = (E->NC > 0 ? ri.comp_end - ri.comp_begin : 0) + tiles;
-            ok = ok && total[r] > 0 && (!solv || tiles > 0);
-            ok_comp = ok_comp && ri.comp_end > ri.comp_begin;
+            total[r] = ri.comp_end - ri.comp_begin + (solv ? ri.stile_end - ri.stile_begin : 0);
+            E->thermo_ok = E->thermo_ok && total[r] > 0;
         }
         E->thermo_total.upload(total);
-        E->thermo_ok_comp = ok_comp;
         E->thermo_cnt.alloc(nsys); E->thermo_cnt.zero();
-        E->thermo_ok = ok;
     }
     E->energy.alloc((size_t)nsys * kEnergyTerms); E->energy.zero();
     E->err.alloc(4); E->err.zero();
@@ -2397,16 +2389,12 @@ int lima_get_config(lima_engine* E, int32_t* out, int32_t n_out) {
         for (const ReplicaInfo& ri : E->reps_h) chunk = std::max(chunk, E->chunk_target(ri));
         const int32_t v[12] = {E->cfg.spt, chunk, (int32_t)E->scwork_h.size(), E->kmax, E->cfg.use_graph,
                                E->n_cells, E->n_stiles, E->R, E->cfg.listed_grid > 0 ? E->cfg.listed_grid : 2 * E->listed_blocks(),
-                               E->cfg.listed_lanes > 0 ? E->cfg.listed_lanes : 4, E->listed_form(), E->thermo_form()};
+                               E->cfg.listed_lanes, E->listed_form(), E->thermo_form()};
         for (int i = 0; i < std::min<int32_t>(n_out, 12); i++) out[i] = v[i];
         return LIMA_OK;
     });
 }
 
-// Autotuner: picks the all-pairs kernel's solvents per thread and chunk size, and
-// the listed kernel's grid, by timing each candidate alone on the current state
-// (state and lists are not modified).  Results are cached per shape histogram in
-// the process and, when LIMA_AUTOTUNE_CACHE names a file, across processes.
 int lima_set_kernel_clock(lima_engine* E, int32_t on) {
     return guarded(E, [&] {
         HIP_TRY(hipSetDevice(E->device));
@@ -2442,6 +2430,9 @@ int lima_get_kernel_clock(lima_engine* E, double* total_us, int64_t* launches) {
     });
 }
 
+// Autotuner: picks the all-pairs role's chunk size, the listed compound role's grid and form, and where the
+// thermostat runs, by timing whole steps of each from the current state, which is restored.  Results are
+// cached per shape histogram in the process and, when LIMA_AUTOTUNE_CACHE names a file, across processes.
 int lima_autotune(lima_engine* E, int32_t reps) {
     return guarded(E, [&] {
         if (reps <= 0) reps = 10;
@@ -2457,7 +2448,7 @@ int lima_autotune(lima_engine* E, int32_t reps) {
             if (it != g_tune_cache.end()) { best = it->second; have = true; }
         }
         if (!have) {
-            // Each shape is timed on the whole step: captured cycles of all streams, rebuilds
+            // Each shape is timed on the whole step: captured cycles, rebuilds
             // included, from the same saved state, which is restored afterwards.  Isolated kernel
             // timings ranked the all-pairs chunk sizes differently from the step they run in.
             hipEvent_t e0, e1;
@@ -2522,76 +2513,62 @@ int lima_autotune(lima_engine* E, int32_t reps) {
             // picked while a slow listed form dominates the step can be the wrong one once it is gone)
             auto sweep_all_pairs = [&] {
                 if (!(E->params.enable_solvents && E->NS > 0 && E->NCH > 0)) return;
-                const int spts[1] = {1}, chunks[4] = {256, 512, 1024, 2048};
-                double tmin[1][4];
-                for (auto& row : tmin)
-                    for (double& v : row) v = 1e30;
+                const int chunks[4] = {256, 512, 1024, 2048};
+                double tmin[4] = {1e30, 1e30, 1e30, 1e30};
                 for (int sweep = 0; sweep < kSweeps; sweep++) {
-                    for (int i = 0; i < 1; i++) {
-                        for (int j = 0; j < 4; j++) {
-                            E->cfg.spt = spts[i];
-                            E->cfg.chunk_particles = chunks[j];
-                            tmin[i][j] = std::min(tmin[i][j], trial());
-                        }
+                    for (int j = 0; j < 4; j++) {
+                        E->cfg.chunk_particles = chunks[j];
+                        tmin[j] = std::min(tmin[j], trial());
                     }
                 }
-                double tbest = 1e30;
-                for (int i = 0; i < 1; i++)
-                    for (int j = 0; j < 4; j++)
-                        if (tmin[i][j] < tbest) { tbest = tmin[i][j]; best.spt = spts[i]; best.chunk_particles = chunks[j]; }
+                const double tbest = *std::min_element(tmin, tmin + 4);
                 // shapes within 2% of the best step are ties at the trials' resolution (repeated
                 // whole-step trials of one shape spread by about that much).  Among them, those
-                // whose all-pairs kernel alone is within 5% of the fastest (a shape with too few
-                // work items to fill the device alone leaves the step to the concurrent streams
+                // whose all-pairs role alone is within 5% of the fastest (a shape with too few
+                // work items to fill the device alone leaves the step to the other roles
                 // at this size and may not at another), and of those the one writing the fewest
-                // per-chunk partials (less HBM traffic, fewer blocks beside the other streams;
+                // per-chunk partials (less HBM traffic, fewer blocks beside the other roles;
                 // shapes that differ only in chunking run within a few per cent alone), then the
                 // fastest alone
-                double kms[1][4];
-                long long parts[1][4];
+                double kms[4];
+                long long parts[4];
                 double kbest = 1e30;
-                for (int i = 0; i < 1; i++)
-                    for (int j = 0; j < 4; j++) {
-                        kms[i][j] = 1e30;
-                        parts[i][j] = 0;
-                        if (tmin[i][j] > 1.02 * tbest) continue;
-                        E->cfg.spt = spts[i];
-                        E->cfg.chunk_particles = chunks[j];
-                        E->build_scwork();
-                        E->reps.upload(E->reps_h);
-                        for (int r = 0; r < E->R; r++)
-                            parts[i][j] += (long long)E->reps_h[r].chunk_count *
-                                           (E->reps_h[r].solv_end - E->reps_h[r].solv_begin);
-                        StepArgs ka = E->step_args(E->cur);
-                        ka.kclock = nullptr;
-                        auto launch = [&] {
-                            if (E->params.accumulation == LIMA_ACCUM_FIXED64) E->launch_roles<true, false>(ka, lima_engine::kRoleAllPairs);
-                            else E->launch_roles<false, false>(ka, lima_engine::kRoleAllPairs);
-                        };
-                        launch();
-                        HIP_TRY(hipEventRecord(e0, E->stream));
-                        for (int k = 0; k < 5; k++) launch();
-                        HIP_TRY(hipEventRecord(e1, E->stream));
-                        HIP_TRY(hipEventSynchronize(e1));
-                        float ms = 0;
-                        HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
-                        kms[i][j] = ms;
-                        kbest = std::min(kbest, (double)ms);
-                    }
+                for (int j = 0; j < 4; j++) {
+                    kms[j] = 1e30;
+                    parts[j] = 0;
+                    if (tmin[j] > 1.02 * tbest) continue;
+                    E->cfg.chunk_particles = chunks[j];
+                    E->build_scwork();
+                    E->reps.upload(E->reps_h);
+                    for (int r = 0; r < E->R; r++)
+                        parts[j] += (long long)E->reps_h[r].chunk_count * (E->reps_h[r].solv_end - E->reps_h[r].solv_begin);
+                    StepArgs ka = E->step_args(E->cur);
+                    ka.kclock = nullptr;
+                    auto launch = [&] {
+                        if (E->params.accumulation == LIMA_ACCUM_FIXED64) E->launch_roles<true, false>(ka, lima_engine::kRoleAllPairs);
+                        else E->launch_roles<false, false>(ka, lima_engine::kRoleAllPairs);
+                    };
+                    launch();
+                    HIP_TRY(hipEventRecord(e0, E->stream));
+                    for (int k = 0; k < 5; k++) launch();
+                    HIP_TRY(hipEventRecord(e1, E->stream));
+                    HIP_TRY(hipEventSynchronize(e1));
+                    float ms = 0;
+                    HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+                    kms[j] = ms;
+                    kbest = std::min(kbest, (double)ms);
+                }
                 long long pbest = -1;
                 double kpick = 1e30;
-                for (int i = 0; i < 1; i++)
-                    for (int j = 0; j < 4; j++) {
-                        if (kms[i][j] > 1.05 * kbest) continue;   // not a step tie, or slow alone
-                        if (pbest < 0 || parts[i][j] < pbest || (parts[i][j] == pbest && kms[i][j] < kpick)) {
-                            pbest = parts[i][j];
-                            kpick = kms[i][j];
-                            best.spt = spts[i];
-                            best.chunk_particles = chunks[j];
-                        }
+                for (int j = 0; j < 4; j++) {
+                    if (kms[j] > 1.05 * kbest) continue;   // not a step tie, or slow alone
+                    if (pbest < 0 || parts[j] < pbest || (parts[j] == pbest && kms[j] < kpick)) {
+                        pbest = parts[j];
+                        kpick = kms[j];
+                        best.chunk_particles = chunks[j];
                     }
+                }
                 restore();
-                E->cfg.spt = best.spt;
                 E->cfg.chunk_particles = best.chunk_particles;
             };
             sweep_all_pairs();
@@ -2621,25 +2598,18 @@ int lima_autotune(lima_engine* E, int32_t reps) {
                 E->cfg.listed_grid = best.listed_grid;
                 E->cfg.listed_packed = best.listed_packed;
             }
-            if (E->thermo_ok || E->thermo_ok_comp) {
-                // the thermostat as its own kernel after the integrators, or in their last blocks: that
-                // saves a launch, but each counting block then releases its partial at device scope,
-                // which writes back its XCD's L2 while other kernels may still run (form 1, both
-                // integrators count); form 2 counts in the compound integrator only, run after the
-                // solvent one
-                const bool offer[3] = {true, E->thermo_ok, E->thermo_ok_comp};
-                double fmin[3] = {1e30, 1e30, 1e30};
+            if (E->thermo_ok) {
+                // the thermostat as its own kernel (between the steps of a graph, beside the next one's
+                // forces), or in the integrate launch's last blocks: that saves its launch, but every
+                // integrator block then releases its partial at device scope, which writes back its XCD's L2
+                double fmin[2] = {1e30, 1e30};
                 for (int sweep = 0; sweep < kSweeps; sweep++) {
-                    for (int j = 0; j < 3; j++) {
-                        if (!offer[j]) continue;
+                    for (int j = 0; j < 2; j++) {
                         E->cfg.fused_thermostat = j;
                         fmin[j] = std::min(fmin[j], trial());
                     }
                 }
-                int jb = 0;
-                for (int j = 1; j < 3; j++)
-                    if (fmin[j] < fmin[jb]) jb = j;
-                best.fused_thermostat = jb;
+                best.fused_thermostat = fmin[1] < fmin[0] ? 1 : 0;
                 E->cfg.fused_thermostat = best.fused_thermostat;
             }
             sweep_all_pairs();
@@ -2647,7 +2617,6 @@ int lima_autotune(lima_engine* E, int32_t reps) {
             (void)hipEventDestroy(e1);
             // choices that the systems did not offer (no solvents, no compounds) are kept as what the engine runs
             if (best.chunk_particles <= 0) best.chunk_particles = 1024;
-            if (best.listed_lanes <= 0) best.listed_lanes = 4;
             if (best.listed_packed < 0) best.listed_packed = E->listed_form();
             std::lock_guard<std::mutex> lk(g_tune_mu);
             g_tune_cache[key] = best;
