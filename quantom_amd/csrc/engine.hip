@@ -1859,7 +1859,9 @@ int io_layout(lima_engine* E, const IoArray (&io)[4], IoArrays& a) {
         a.p[k] = io[k].dev;
         a.end[k] = (int)(total += io[k].host ? io[k].n : 0);
     }
-    if (total && total * 12 <= kIoPinned && !E->io_pinned) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&E->io_pinned), kIoPinned, 0));
+    // as large as all four arrays of this engine need: a batch of small engines keeps as many buffers
+    if (total && total * 12 <= kIoPinned && !E->io_pinned)
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&E->io_pinned), std::min(kIoPinned, E->io_dev.n * sizeof(float)), 0));
     return (int)total;
 }
 void io_get(lima_engine* E, const IoArray (&io)[4]) {

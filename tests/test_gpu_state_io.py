@@ -69,3 +69,25 @@ def test_state_and_forces_take_no_device_memory(small_system):
     assert free() == before
     e.close()
     f.close()
+
+
+def test_small_engines_keep_small_transfer_buffers(small_system):
+    """32 engines of 78 KB of state each: their first reading of it takes less than 1 MB of the
+    process's address space an engine (pinned memory is mapped into it)."""
+    from quantom_amd.abi import RunParams
+    from quantom_amd.engine import Engine
+
+    def mapped():
+        with open("/proc/self/status") as f:
+            return next(int(line.split()[1]) for line in f if line.startswith("VmSize"))
+
+    first = Engine([small_system], RunParams())
+    first.get_state()
+    engines = [Engine([small_system], RunParams()) for _ in range(32)]
+    before = mapped()
+    for e in engines:
+        e.get_state()
+    grown = mapped() - before
+    assert grown < 32 * 1024, grown
+    for e in engines + [first]:
+        e.close()
