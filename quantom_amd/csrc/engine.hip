@@ -2509,6 +2509,11 @@ int lima_autotune(lima_engine* E, int32_t reps) {
                     timed = std::max(timed, (want + cyc - 1) / cyc * cyc);
                 }
             }
+            // the chunk size that every system has by its own size, or 0
+            int own_chunk = -1;
+            E->cfg.chunk_particles = 0;
+            for (const ReplicaInfo& ri : E->reps_h)
+                own_chunk = own_chunk < 0 || own_chunk == E->chunk_target(ri) ? E->chunk_target(ri) : 0;
             // three sweeps, the fastest time of each shape (clocks ramp after idle periods)
             constexpr int kSweeps = 3;
             // the all-pairs shape, swept again after the listed kernels' choices below (a shape
@@ -2524,21 +2529,21 @@ int lima_autotune(lima_engine* E, int32_t reps) {
                     }
                 }
                 const double tbest = *std::min_element(tmin, tmin + 4);
-                // shapes within 2% of the best step are ties at the trials' resolution (repeated
-                // whole-step trials of one shape spread by about that much).  Among them, those
+                // shapes within 1% of the best step are ties at the trials' resolution.  Among them, the
+                // chunk that the engine takes untuned (the 256 replicas took 512 over their own 256, equal
+                // in the trials, 1.3% slower over 60 steps and 2.3% over 2,000).  Else, of those
                 // whose all-pairs role alone is within 5% of the fastest (a shape with too few
                 // work items to fill the device alone leaves the step to the other roles
-                // at this size and may not at another), and of those the one writing the fewest
-                // per-chunk partials (less HBM traffic, fewer blocks beside the other roles;
-                // shapes that differ only in chunking run within a few per cent alone), then the
-                // fastest alone
+                // at this size and may not at another), the one writing the fewest
+                // per-chunk partials (less HBM traffic; shapes that differ only in chunking run
+                // within a few per cent alone), then the fastest alone
                 double kms[4];
                 long long parts[4];
                 double kbest = 1e30;
                 for (int j = 0; j < 4; j++) {
                     kms[j] = 1e30;
                     parts[j] = 0;
-                    if (tmin[j] > 1.02 * tbest) continue;
+                    if (tmin[j] > 1.01 * tbest) continue;
                     E->cfg.chunk_particles = chunks[j];
                     E->build_scwork();
                     E->reps.upload(E->reps_h);
@@ -2570,6 +2575,8 @@ int lima_autotune(lima_engine* E, int32_t reps) {
                         best.chunk_particles = chunks[j];
                     }
                 }
+                for (int j = 0; j < 4; j++)
+                    if (chunks[j] == own_chunk && tmin[j] <= 1.01 * tbest) best.chunk_particles = own_chunk;
                 restore();
                 E->cfg.chunk_particles = best.chunk_particles;
             };
