@@ -349,16 +349,17 @@ struct lima_engine {
         return a;
     }
 
-    // solvent list row stride: capacity rounded up to 4 ints (16-byte aligned rows)
+    // solvent list row stride: capacity rounded up to the 16 ids that a quad reads at a time
     int ss_ld() const { return (params.max_solvent_neighbors + kListChunk - 1) / kListChunk * kListChunk; }
 
     // ---- launches ----
     // Target rows of a system's all-pairs chunks.  The sums of a chunk are added to the next one's,
     // so the choice depends on the system alone and not on what is batched with it: 1024 rows where
-    // that leaves about one block a wavefront slot (1000 of 256 threads), else smaller chunks down
-    // to 128 rows.  Alone: 36 tiles x 2,700 particles 51.7 us at 1024 (120 blocks), 18.4 at 128;
-    // the demo 53.2 and 10.5; production (1,235 blocks at 1024) gains nothing from smaller ones, the
-    // 18 nm box loses 9% at 128 (the rows' staging).
+    // that leaves about one block a wavefront slot (1000 of 256 threads), else 512 or 256.  Alone, us,
+    // at 1024, 512 and 256 rows: 46 tiles x 2,700 particles 46.7, 24.6, 17.2; the demo 49.8, 26.2, 14.6;
+    // production (1,235 blocks at 1024) 121, 116, 110, where its step is the shortest at 1024; the
+    // 18 nm box 2,552, 2,575, 2,675 (the rows' staging).  128 rows gained small systems 2-3% and cost
+    // batches as much.
     int chunk_target(const ReplicaInfo& ri) const {
         if (cfg.chunk_particles > 0) return std::min(cfg.chunk_particles, kChunkParticles);
         const int tiles = (ri.solv_end - ri.solv_begin + kStepThreads - 1) / kStepThreads;

@@ -83,16 +83,16 @@ struct StepArgs {
     float4* ss_img;               // the solvent's position after the reference's re-imaging sequence
     const int* cw_off; const int* cw_total;
     const int* item_comp;         // [work item] its compound (written with cw_off at each rebuild)
-    const int* run_off; const int* run_cs_off; const int* run_total; const int* run_comp;   // packed listed kernel's runs
+    const int* run_off; const int* run_cs_off; const int* run_total; const int* run_comp;   // listed_packed_role's runs
     const float2* tab_inter_ab;   // [R*1024] lj_ab of tab_inter, [source type * 32 + target type]
     const float2* tab_intra_ab;   // [R*1024] lj_ab of tab_intra
     // partial forces
     float4* partC;  I3* partC_fx;   // [slot*128 + p]
-    float4* cloc;   I3* cloc_fx;    // [n_chain] bridge + bonded + intra-compound LJ (compound_local_kernel)
+    float4* cloc;   I3* cloc_fx;    // [n_chain] bonded + intra-compound LJ (local_role); the integrator adds the bridges'
     float4* partS;  I3* partS_fx;   // [chunk*n_solv + s]
     const SCWork* scwork; int n_scwork;
     int chunk_cap;                // rows of the largest solvent<-chain chunk (LDS tile size)
-    const int* comp_row;          // [n_comp+1] first row of each compound in the all-pairs kernel's tiles (multiples of kRowPad)
+    const int* comp_row;          // [n_comp+1] first row of each compound in all_pairs_role's tiles (multiples of kRowPad)
     const int* row_src;           // [rows] chain particle of each row, -1: padding
     // thermostat
     const float* lambda;          // [R] applied this step
@@ -113,7 +113,7 @@ struct StepArgs {
     double* temperature;          // [R]
     long long* step_count_w;      // [R] the step counters (the thermostat advances them)
     int thermo_mode;
-    unsigned long long* kclock;   // [4] span of the step's solvent_chain_kernel and its running sum, or null
+    unsigned long long* kclock;   // [4] span of the step's all-pairs blocks and its running sum, or null
     float* log_data;              // [log_ring][10]
     float* train_data;            // [log_ring][compounds of log_rep][log_slots][3 x Float3], or null
     // energies: [R*kEnergyTerms]
@@ -495,7 +495,7 @@ LIMA_DEV bool in_box(float4 p, float L) {
     return p.x >= 0.f && p.x <= L && p.y >= 0.f && p.y <= L && p.z >= 0.f && p.z <= L;
 }
 
-// In-step timing of the all-pairs kernel, on the device's constant-rate clock (wall_clock64):
+// In-step timing of all_pairs_role, on the device's constant-rate clock (wall_clock64):
 // kclock[0] = the earliest start of the first kClockHead blocks (dispatched first, one per
 // XCD), kclock[1] = the latest end of any block (work items differ in length, so any block
 // may be the last); the step's thermostat kernel, which runs after it on the same stream,
@@ -867,8 +867,8 @@ LIMA_DEV void listed_role(const StepArgs& a, int blk, int nblk, char* lds) {
 // 256 sources staged and summed in two halves of 128), or up to cc_run(PPL) = 8 / PPL
 // consecutive neighbour-compound items of one compound (at most 128 sources, staged together).
 // Lane pi of a group holds particles pi, pi + 16, ... of the run's compound and sums each
-// item's sources whole in list order, so every work item is still one sequential sum per
-// particle written to its own partial slot, as in listed_role.  A group reads only
+// item's sources in list order, in the parts that listed_role sums them in, into the item's
+// own partial slot: the sums are the same.  A group reads only
 // its own LDS row, so wavefront-level ordering is the only synchronisation.  Groups may belong
 // to different replicas: the inter-compound pair constants come from a table of the used types in
 // LDS when every group is of the system of the block's first run, else from the global table
@@ -1387,7 +1387,7 @@ LIMA_DEV void thermostat_replica(int r, const ReplicaInfo& rp, int lane, const d
         lambda_applied[r] = lambda[r];
         const long long done = step_count[r] + 1;
         step_count[r] = done;
-        if (kclock && r == 0) {   // this step's span of the all-pairs kernel
+        if (kclock && r == 0) {   // this step's span of the all-pairs blocks
             const unsigned long long b = kclock[0], e = kclock[1];
             if (b != ~0ull && e > b) {
                 kclock[2] += e - b;
@@ -1713,7 +1713,7 @@ template <bool ADVANCE, bool FIXED, bool ENERGY, int SLOTS> LIMA_DEV void compou
             }
             if (cl == 0 && p == 0) {
                 // outdata of compound 0, particle 0 (Engine.cu:1019-1028): speed, kinetic energy of the
-                // one-step-apart positions, |F| (thread 0's potE slot comes from compound_local_kernel)
+                // one-step-apart positions, |F| (thread 0's potE slot comes from local_role)
                 float bx = qx, by = qy, bz = qz;
                 hyperpos(px, py, pz, bx, by, bz, box);
                 float* o = a.log_data + (size_t)ring * 10;
@@ -1863,7 +1863,7 @@ struct NlistArgs {
     int max_segs;
     int* cw_off; int* cw_total;
     int* item_comp;
-    int run_len;                  // neighbour items per run of the packed listed kernel (0: not used)
+    int run_len;                  // neighbour items per run of listed_packed_role (0: not used)
     int* run_off; int* run_cs_off; int* run_total; int* run_comp;   // run_total[2]: neighbour runs, solvent chunks
     uint32_t* err;
     int enable_solvents;
@@ -2285,7 +2285,7 @@ __global__ __launch_bounds__(kSolventListThreads) void nl_solvent_solvent_kernel
 }
 
 // per compound work slots: listed neighbours + ceil(solvent list / 256); exclusive scan.  With
-// run_len > 0 (the packed listed kernel), also the compound's runs: ceil(neighbours / run_len)
+// run_len > 0 (listed_packed_role), also the compound's runs: ceil(neighbours / run_len)
 // + ceil(solvent list / 256), scanned into run_off.
 // run_len > 0: the compound's runs of run_len neighbours; run_len == 0: its work items (one per
 // listed neighbour, then one per solvent chunk); run_len < 0: its solvent chunks alone
@@ -2329,7 +2329,7 @@ LIMA_DEV void nl_items(const NlistArgs& a, int c, int lane) {
         for (int w = a.run_cs_off[c] + lane; w < a.run_cs_off[c + 1]; w += 64) a.run_comp[cs0 + w] = c;
     }
 }
-// With run_len > 0 (the packed listed kernel) the run list holds every compound's neighbour
+// With run_len > 0 (listed_packed_role) the run list holds every compound's neighbour
 // runs first (run_off, run_total[0] of them), then every compound's solvent chunks (run_cs_off,
 // run_total[1]), so that the groups of a wavefront mostly take runs of one kind.
 __global__ __launch_bounds__(1024) void nl_work_kernel(NlistArgs a) {
