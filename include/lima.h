@@ -268,8 +268,9 @@ int lima_get_kernel_clock(lima_engine* engine, double* total_us, int64_t* launch
    the listed compound role for compounds of at most 64 particles (1 packed,
    2 (FP32) plain with the sources of compounds of at most 32 particles split
    over both halves of a wavefront, else 0), and where the thermostat runs: 0 after
-   the integrators (a kernel of its own, or beside the next step's forces), 1 or 2
-   the last integrator block of each system (same sums in all). */
+   the integrators (a kernel of its own, or beside the next step's forces), 1 in
+   the last integrator block of each system (2 if a saved tuning says so, the same);
+   the sums are the same. */
 int lima_get_config(lima_engine* engine, int32_t* out, int32_t n_out);
 /* Picks the launch shape (chunk size of the all-pairs role, grid and form of the
    listed compound role, where the thermostat runs) by timing whole steps of each shape,
